@@ -407,13 +407,14 @@ constexpr int spectral_modes_per_block(int lpm, int e, bool mixed)
 }
 // waves per SIMD that the LDS of one CU (160 KiB) allows, at most 3: the
 // lane-group solve needs 136 (E = 2) to 226 (E = 8) VGPRs, and a tighter
-// register cap sends it to scratch
+// register cap sends it to scratch (at 4: 44, 80 and 140 bytes per lane for
+// 8 x 2, 16 x 2 and 16 x 4, where 3 leaves none)
 constexpr int spectral_waves_per_simd(int lpm, int e, bool mixed)
 {
   const int G = spectral_modes_per_block(lpm, e, mixed);
   const int blocks = (int)(163840 / spectral_lds_bytes(lpm, e, G, mixed));
   const int w = blocks * (G * lpm / 64) / 4;
-  return w < 1 ? 1 : (w > 4 ? 4 : w);
+  return w < 1 ? 1 : (w > 3 ? 3 : w);
 }
 void launch_bvp_factor(const BvpConsts& B, const double* ksq, int nk, double* s_ib, double* s_ab, int lpm,
                        int e, double* fib, double* fab, double* fG, hipStream_t s);

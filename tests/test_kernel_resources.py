@@ -1,0 +1,57 @@
+"""Private memory of the built kernels (from the metadata of the gfx950 code
+objects in the library): the FP32 lane-group spectral solve of up to 32 and
+of 49 to 64 levels keeps its rows in registers, none of them in scratch."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+from doublyperiodicstokes_amd import build as b
+
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def code_objects(data):
+    """The gfx950 ELF images of every offload bundle in the library."""
+    at = data.find(MAGIC)
+    while at >= 0:
+        n, = struct.unpack_from("<Q", data, at + len(MAGIC))
+        p = at + len(MAGIC) + 8
+        for _ in range(n):
+            off, size, tl = struct.unpack_from("<QQQ", data, p)
+            triple = data[p + 24:p + 24 + tl]
+            p += 24 + tl
+            if b"gfx950" in triple and size:
+                yield data[at + off:at + off + size]
+        at = data.find(MAGIC, at + 1)
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{demangled kernel name: scratch bytes per lane}."""
+    llvm = os.path.join(b.ROCM, "llvm", "bin")
+    tool = os.path.join(llvm, "llvm-readelf")
+    if not os.path.exists(b.lib_path()):
+        b.build()
+    if not os.path.exists(tool):
+        pytest.skip("llvm-readelf not found")
+    d = tmp_path_factory.mktemp("co")
+    out = {}
+    with open(b.lib_path(), "rb") as f:
+        data = f.read()
+    for i, image in enumerate(code_objects(data)):
+        path = d / ("%d.co" % i)
+        path.write_bytes(image)
+        text = subprocess.run([tool, "--notes", str(path)], stdout=subprocess.PIPE, check=True).stdout.decode()
+        for m in re.finditer(r"\.name:\s+(_Z\S*)\n\s+\.private_segment_fixed_size:\s+(\d+)", text):
+            out[m.group(1)] = int(m.group(2))
+    return out
+
+
+@pytest.mark.parametrize("lpm,e", [(8, 2), (16, 2), (16, 4)])
+def test_lane_group_solve_has_no_scratch(kernels, lpm, e):
+    found = [v for k, v in kernels.items() if "k_spectralIfLi%dELi%dE" % (lpm, e) in k]
+    assert len(found) == 1
+    assert found[0] == 0
