@@ -325,8 +325,12 @@ void fft_x_launch(const void* in, void* out, int nrows, const void* tw, int dir,
 // Other lengths N = R1 R2 with radices of 1 .. 35 points (products of 2, 3, 5
 // and 7): the same two passes with the radices chosen at run time, each pass a
 // switch over its register transforms.  RMAX bounds the radices a kernel holds
-// (its registers are those of the largest): 10, 16 or 35 (180 x 140 x 65 mixed,
-// both directions: 57 us, with the 35-point kernels for all lengths 65).  Bound by
+// (its registers are those of the largest): 10, 16, 20 or 35 (180 x 140 x 65 mixed,
+// both directions: 57 us, with the 35-point kernels for all lengths 65).  In FP64
+// the strided 35-point kernels need scratch (456 bytes per lane), which made the
+// even lengths of radices 18 and 20 slower than rocFFT: 162^2 x 40 85 us against 73,
+// 200^2 97 / 84, 216^2 121 / 96; with kernels of their own 73, 87 and 105, and
+// 270^2 148 -> 130, 400^2 303 -> 271 (rocFFT 157 and 467).  Bound by
 // memory and its latency, as k_fft_y; rocFFT with its transposes and separate
 // pre- and post-processing kernels took 104 us there, 67 against 47 at 160^2 x 57,
 // and 90 against 48 for the triply periodic 96^3.
@@ -652,6 +656,7 @@ void launch_fft_x(const void* in, void* out, int nrows, int Nx, const void* tw, 
       if (!split_length(Nx, &R1, &R2)) return;   // callers check fft_x_supported
       if (R1 <= 10) rows_launch<T, 10>(in, out, nrows, R1, R2, tw, dir, s);
       else if (R1 <= 16) rows_launch<T, 16>(in, out, nrows, R1, R2, tw, dir, s);
+      else if (R1 <= 20) rows_launch<T, 20>(in, out, nrows, R1, R2, tw, dir, s);
       else rows_launch<T, 35>(in, out, nrows, R1, R2, tw, dir, s);
     }
   }
@@ -686,6 +691,7 @@ void launch_fft_y(void* data, int nslices, int Nkx, int Ny, const void* tw, int 
       if (!split_length(Ny, &R1, &R2)) return;   // callers check fft_y_supported
       if (R1 <= 10) cols_launch<T, 10>(data, nslices, Nkx, R1, R2, tw, dir, s);
       else if (R1 <= 16) cols_launch<T, 16>(data, nslices, Nkx, R1, R2, tw, dir, s);
+      else if (R1 <= 20) cols_launch<T, 20>(data, nslices, Nkx, R1, R2, tw, dir, s);
       else cols_launch<T, 35>(data, nslices, Nkx, R1, R2, tw, dir, s);
     }
   }

@@ -1,6 +1,7 @@
 """Private memory of the built kernels (from the metadata of the gfx950 code
 objects in the library): the FP32 lane-group spectral solve of up to 32 and
-of 49 to 64 levels keeps its rows in registers, none of them in scratch."""
+of 49 to 64 levels keeps its rows in registers, none of them in scratch, and
+so do the FFT kernels for radices up to 20 in both precisions."""
 import os
 import re
 import struct
@@ -55,3 +56,11 @@ def test_lane_group_solve_has_no_scratch(kernels, lpm, e):
     found = [v for k, v in kernels.items() if "k_spectralIfLi%dELi%dE" % (lpm, e) in k]
     assert len(found) == 1
     assert found[0] == 0
+
+
+@pytest.mark.parametrize("real", ["f", "d"])
+@pytest.mark.parametrize("rmax", [10, 16, 20])
+def test_fft_kernels_have_no_scratch(kernels, real, rmax):
+    for name in ("k_fft_colsI%sLi%dELin1E", "k_fft_colsI%sLi%dELi1E", "k_fft_rows_fwdI%sLi%dE", "k_fft_rows_invI%sLi%dE"):
+        found = [v for k, v in kernels.items() if name % (real, rmax) in k]
+        assert found == [0], name
