@@ -126,9 +126,21 @@ struct dps_handle {
   // and tile order, rebuilt whenever positions change
   int list_cap = 0;
   int *d_lcounts = nullptr, *d_lstart = nullptr, *d_lcursor = nullptr, *d_lunsorted = nullptr, *d_lentries = nullptr;
-  // cells of the fixed-point spreading (mixed precision)
-  int *d_fx_counts = nullptr, *d_fx_start = nullptr, *d_fx_entries = nullptr;
-  int fx_cap = 0;
+  // fixed-point spreading of FP64 arrays (mixed precision): the cell lists of
+  // each pass that the solver has (FX_FORCES ...)
+  struct FxLists {
+    int *counts = nullptr, *start = nullptr, *entries = nullptr;
+    int cap = 0;
+  } fx[3];
+  // passes whose lists every locate builds: from a pass's first product on,
+  // which builds them itself (solvers that see FP32 arrays only never do)
+  unsigned fx_on = 0;
+  // passes that a captured locate left out: its replays would leave their lists
+  // behind, so each of their products builds them
+  unsigned fx_lost = 0;
+  // a captured product reads the lists as they are, with its own ZC: ZC stays
+  bool fx_pinned = false;
+  bool in_batch_capture = false;   // (a batch captures again when ZC changes)
   float* d_amax = nullptr;
   int *d_key = nullptr, *d_rank = nullptr, *d_kcounts = nullptr, *d_kstart = nullptr, *d_order = nullptr;
   void* d_grid = nullptr;
@@ -442,14 +454,31 @@ int check_spread_sizes(dps_handle* h)
   if (pm < 0 || pd < 0) return fail(DPS_ERR_ARG, "kernel z support too long for the spreading lists");
   const long most = (h->has_dip && !h->reg && !pair) ? pm + pd : std::max(pm, pd);
   if (h->N * most > (long)INT32_MAX) return fail(DPS_ERR_ARG, "too many spreading entries");
-  h->fx_cap = (int)std::max(1L, h->N * most);
   return DPS_OK;
 }
 
-void set_chunk(dps_handle* h, int zc)
+// tiles of T points that a run of w of n points meets at most; periodic: the
+// last tile may be short and the run may cross the end
+int run_tiles_bound(int w, int T, int n, bool periodic)
 {
-  h->ZC = zc;
-  h->nt = std::max(1, std::min(3, (zc + 15) / 16));
+  return (w + T - 2) / T + 1 + (periodic && n % T ? 1 : 0);
+}
+
+// capacities of the fixed-point cell lists, for the shortest z chunk
+void size_fx_lists(dps_handle* h)
+{
+  const bool tp = h->geometry == DPS_MODE_PERIODIC;
+  const bool pair = h->has_dip && !h->reg && h->km.wx == h->kd.wx && h->km.wy == h->kd.wy;
+  auto per = [&](const KernelDesc& K, int S) {
+    return (long)run_tiles_bound(K.wx, FX_TX, h->Nx, true) * run_tiles_bound(K.wy, FX_TY, h->Ny, true) *
+           run_tiles_bound(S, h->zc_min, h->Nz, tp);
+  };
+  auto cap = [&](long n) { return (int)std::max(1L, (long)h->N * n); };   // check_spread_sizes bounds it
+  h->fx[FX_FORCES].cap = cap(per(h->km, h->km.wzmax));
+  if (h->has_dip && h->reg) h->fx[FX_REGULAR].cap = cap(per(h->kd, h->kd.wzmax));
+  if (h->has_dip && !h->reg)
+    h->fx[FX_TORQUES].cap = cap(pair ? per(h->km, h->km.wzmax + h->kd.wzmax)
+                                     : per(h->km, h->km.wzmax) + per(h->kd, h->kd.wzmax));
 }
 
 // spreading tiles and particle records (both z grids)
@@ -514,9 +543,13 @@ int allocate(dps_handle* h)
     if (h->prec == DPS_PREC_MIXED) {
       const size_t ncells = (size_t)((h->Nx + FX_TX - 1) / FX_TX) * ((h->Ny + FX_TY - 1) / FX_TY) *
                             ((h->Nz + h->zc_min - 1) / h->zc_min);
-      if ((rc = h->alloc(&h->d_fx_counts, ncells))) return rc;
-      if ((rc = h->alloc(&h->d_fx_start, ncells + 1))) return rc;
-      if ((rc = h->alloc(&h->d_fx_entries, h->fx_cap))) return rc;
+      size_fx_lists(h);
+      for (auto& L : h->fx) {
+        if (!L.cap) continue;
+        if ((rc = h->alloc(&L.counts, ncells))) return rc;
+        if ((rc = h->alloc(&L.start, ncells + 1))) return rc;
+        if ((rc = h->alloc(&L.entries, L.cap))) return rc;
+      }
       if ((rc = h->alloc(&h->d_amax, 2 * FX_AMAX_BLOCKS))) return rc;
     }
     // counts and range flags are zero between builds (k_scan_counts)
@@ -946,6 +979,86 @@ ListArgs list_args(dps_handle* h)
   return A;
 }
 
+// a fixed-point pass of FP64 arrays onto the FP32 grid: forces, forces and
+// torques, or (regular) the torques as a vector field into d_gridT
+FxArgs fx_args(dps_handle* h, int pass)
+{
+  const bool regular = pass == FX_REGULAR, torques = pass == FX_TORQUES;
+  const KernelDesc& K0 = regular ? h->kd : h->km;
+  FxArgs A{};
+  A.N = h->N; A.Nx = h->Nx; A.Ny = h->Ny; A.Nz = h->Nz;
+  A.periodic_z = h->geometry == DPS_MODE_PERIODIC;
+  A.ZC = h->ZC;
+  A.ntx = (h->Nx + FX_TX - 1) / FX_TX;
+  A.nty = (h->Ny + FX_TY - 1) / FX_TY;
+  A.nch = (h->Nz + h->ZC - 1) / h->ZC;
+  A.pair = torques && interp_pairable(h);
+  A.nkind = torques && !A.pair ? 2 : 1;
+  A.wx0 = K0.wx; A.wy0 = K0.wy; A.W0 = K0.wzmax;
+  A.sup0 = regular ? h->d_sup_d : h->d_sup_m;
+  A.sup1 = h->d_sup_d;
+  A.rec = regular ? h->rec_d() : h->d_rec;
+  A.rs = h->rec_stride;
+  A.off1 = h->rec_off_d;
+  A.pm = A.wx0 + A.wy0 + A.W0;
+  if (torques) {
+    A.wx1 = h->kd.wx; A.wy1 = h->kd.wy; A.W1 = h->kd.wzmax;
+    A.pd = 2 * (A.wx1 + A.wy1 + A.W1);
+  }
+  A.ho = A.pair ? A.pm + A.pd : single_words(h);
+  A.counts = h->fx[pass].counts; A.start = h->fx[pass].start; A.entries = h->fx[pass].entries;
+  A.cap = h->fx[pass].cap;
+  A.amax = h->d_amax;
+  A.K0 = 3 * K0.inv_norm3;
+  A.K1 = h->has_dip && !regular ? 3 * h->kd.dmax * h->kd.inv_norm3 : 0.0;
+  A.grid = regular ? h->d_gridT : h->d_grid;
+  return A;
+}
+
+// whether launches on s are being recorded
+bool capturing(hipStream_t s)
+{
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();   // the null stream beside a capture
+  return st != hipStreamCaptureStatusNone;
+}
+
+// the cell lists of every pass that is on, for the located positions and ZC
+void build_fx_lists(dps_handle* h, hipStream_t s)
+{
+  for (int pass = 0; pass < 3; ++pass)
+    if (h->fx_on >> pass & 1) launch_fx_lists(fx_args(h, pass), s);
+}
+
+// A pass is about to read its cell lists: those that the locate built, or, at
+// a pass's first product (and where a replayed locate leaves them out), built
+// here.  The lists depend on the positions alone, so building them in every
+// product would add four launches to each: 17 to 70 us (products at fixed
+// positions, 64x64x30 and 256x256x96).
+void need_fx_lists(dps_handle* h, int pass, hipStream_t s)
+{
+  const unsigned bit = 1u << pass;
+  const bool cap = capturing(s);
+  if (h->fx_on & bit) {
+    if (cap && !h->in_batch_capture) h->fx_pinned = true;
+    return;
+  }
+  launch_fx_lists(fx_args(h, pass), s);
+  if (!cap && !(h->fx_lost & bit)) h->fx_on |= bit;
+}
+
+// z chunk of the fixed-point cells.  It stays as it is where a captured product
+// reads the lists of the present one, or where s only records.
+int set_fx_chunk(dps_handle* h, int zc, hipStream_t s)
+{
+  if (zc == h->ZC || h->fx_pinned) return DPS_OK;
+  if (h->fx_on && capturing(s)) return DPS_OK;
+  h->ZC = zc;
+  build_fx_lists(h, s);
+  HIPCHK(hipGetLastError());
+  return DPS_OK;
+}
+
 // Supports, records and lists from positions (kernels only).  move: a step of
 // positions kept on the device, by vel if given.  report: a set of positions,
 // whose range flag goes to the host; otherwise the device keeps it.
@@ -968,6 +1081,10 @@ int locate(dps_handle* h, void* positions, int dtype, bool move, const void* vel
   }
   HIPCHK(hipGetLastError());
   launch_lists(A.L, s);
+  if (mixed(h)) {
+    build_fx_lists(h, s);
+    if (capturing(s)) h->fx_lost |= ~h->fx_on;
+  }
   HIPCHK(hipGetLastError());
   return DPS_OK;
 }
@@ -1069,38 +1186,17 @@ bool spread_fits(dps_handle* h, bool torques, int zc)
   return chunk_fits(h, pair ? pair_words(h) : single_words(h), zc);
 }
 
-// fixed-point pass of FP64 arrays onto the FP32 grid: forces, forces and
-// torques, or (regular) the torques as a vector field into d_gridT
-void spread_fx_pass(dps_handle* h, bool torques, bool regular, const void* F, const void* Tq, hipStream_t s)
+// the lists of every pass of a product
+void need_fx_lists_of(dps_handle* h, bool torques, hipStream_t s)
 {
-  const KernelDesc& K0 = regular ? h->kd : h->km;
-  FxArgs A{};
-  A.N = h->N; A.Nx = h->Nx; A.Ny = h->Ny; A.Nz = h->Nz;
-  A.periodic_z = h->geometry == DPS_MODE_PERIODIC;
-  A.ZC = h->ZC;
-  A.ntx = (h->Nx + FX_TX - 1) / FX_TX;
-  A.nty = (h->Ny + FX_TY - 1) / FX_TY;
-  A.nch = (h->Nz + h->ZC - 1) / h->ZC;
-  A.pair = torques && interp_pairable(h);
-  A.nkind = torques && !A.pair ? 2 : 1;
-  A.wx0 = K0.wx; A.wy0 = K0.wy; A.W0 = K0.wzmax;
-  A.sup0 = regular ? h->d_sup_d : h->d_sup_m;
-  A.sup1 = h->d_sup_d;
-  A.rec = regular ? h->rec_d() : h->d_rec;
-  A.rs = h->rec_stride;
-  A.off1 = h->rec_off_d;
-  A.pm = A.wx0 + A.wy0 + A.W0;
-  if (torques) {
-    A.wx1 = h->kd.wx; A.wy1 = h->kd.wy; A.W1 = h->kd.wzmax;
-    A.pd = 2 * (A.wx1 + A.wy1 + A.W1);
-  }
-  A.ho = A.pair ? A.pm + A.pd : single_words(h);
-  A.counts = h->d_fx_counts; A.start = h->d_fx_start; A.entries = h->d_fx_entries;
-  A.cap = h->fx_cap;
-  A.amax = h->d_amax;
-  A.K0 = 3 * K0.inv_norm3;
-  A.K1 = h->has_dip && !regular ? 3 * h->kd.dmax * h->kd.inv_norm3 : 0.0;
-  A.grid = regular ? h->d_gridT : h->d_grid;
+  if (h->reg || !torques) need_fx_lists(h, FX_FORCES, s);
+  if (torques) need_fx_lists(h, h->reg ? FX_REGULAR : FX_TORQUES, s);
+}
+
+void spread_fx_pass(dps_handle* h, int pass, const void* F, const void* Tq, hipStream_t s)
+{
+  need_fx_lists(h, pass, s);
+  const FxArgs A = fx_args(h, pass);
   launch_spread_fx(A, staged_words(A.pair ? pair_words(h) : single_words(h)), (const double*)F, (const double*)Tq, s);
 }
 
@@ -1112,10 +1208,10 @@ int do_spread(dps_handle* h, const void* F, const void* T, int dtype, hipStream_
   const void* Tq = (T && h->has_dip) ? T : nullptr;
   if (fp64_results(h, dtype)) {
     if (h->reg) {
-      spread_fx_pass(h, false, false, F, nullptr, s);
-      if (Tq) spread_fx_pass(h, false, true, Tq, nullptr, s);
+      spread_fx_pass(h, FX_FORCES, F, nullptr, s);
+      if (Tq) spread_fx_pass(h, FX_REGULAR, Tq, nullptr, s);
     } else {
-      spread_fx_pass(h, Tq != nullptr, false, F, Tq, s);
+      spread_fx_pass(h, Tq ? FX_TORQUES : FX_FORCES, F, Tq, s);
     }
   } else if (h->reg) {
     spread_pass(spread_args(h, false), F, nullptr, mixed(h), dtype, s);
@@ -1803,7 +1899,7 @@ int dps_batch_mdot(dps_batch* b, const void* const* forces, const void* const* t
   if (dtype != DPS_F32 && dtype != DPS_F64) return fail(DPS_ERR_ARG, "dtype must be DPS_F32 or DPS_F64");
   const int n = (int)b->hs.size();
   std::vector<const void*> key;
-  key.reserve(4 * n + 1);
+  key.reserve(5 * n + 1);
   for (int i = 0; i < n; ++i) {
     int rc = check_handle(b->hs[i], true);
     if (rc) return rc;
@@ -1815,11 +1911,18 @@ int dps_batch_mdot(dps_batch* b, const void* const* forces, const void* const* t
     key.push_back(t);
     key.push_back(velocities[i]);
     key.push_back(angular ? angular[i] : nullptr);
+    // launch shapes: another batch of this instance may have changed them
+    key.push_back((const void*)(intptr_t)(1024 * h->ZC + h->nt));
   }
   key.push_back((const void*)(intptr_t)(dtype + 1));
   hipStream_t s = (hipStream_t)stream;
   if (!b->exec || key != b->key) {
     b->drop_graph();
+    // cell lists that no product has asked for yet are built now, not in every replay
+    if (!capturing(s))
+      for (int i = 0; i < n; ++i)
+        if (fp64_results(b->hs[i], dtype)) need_fx_lists_of(b->hs[i], torques && torques[i], s);
+    HIPCHK(hipGetLastError());
     // capturing records no work: capture on the batch's own stream, launch on
     // the caller's
     hipStream_t c = b->cap;
@@ -1832,8 +1935,10 @@ int dps_batch_mdot(dps_batch* b, const void* const* forces, const void* const* t
       dps_handle* h = b->hs[i];
       const bool p = h->prof;
       h->prof = false;   // no timing events inside the graph
+      h->in_batch_capture = true;
       rc = dps_mdot(h, forces[i], torques ? torques[i] : nullptr, velocities[i], angular ? angular[i] : nullptr,
                     dtype, (void*)b->streams[i % ns]);
+      h->in_batch_capture = false;
       h->prof = p;
       h->have_timings = false;
     }
@@ -1903,7 +2008,7 @@ int dps_batch_tune(dps_batch* b, const void* const* forces, const void* const* t
       if (ms < best_ms) { best_ms = ms; best = zc; best_nt = h->nt; }
     }
     h->nt = best_nt;
-    if (best) h->ZC = best;
+    if (best && !rc) rc = set_fx_chunk(h, best, s);
     if (chunk_out) chunk_out[i] = h->ZC;
   }
   (void)hipEventDestroy(e0);
@@ -1916,7 +2021,7 @@ int dps_batch_set_chunks(dps_batch* b, const int* chunks, int torques, void* str
 {
   if (!b) return fail(DPS_ERR_STATE, "null batch");
   if (!chunks) return fail(DPS_ERR_ARG, "null chunks");
-  (void)stream;   // a chunk changes launches only
+  hipStream_t s = (hipStream_t)stream;
   int rc;
   // every instance is checked before any changes, so a refused call leaves
   // the batch as it was
@@ -1930,7 +2035,8 @@ int dps_batch_set_chunks(dps_batch* b, const int* chunks, int torques, void* str
   }
   for (size_t i = 0; i < b->hs.size(); ++i) {
     dps_handle* h = b->hs[i];
-    set_chunk(h, chunks[i]);
+    h->nt = std::max(1, std::min(3, (chunks[i] + 15) / 16));
+    if ((rc = set_fx_chunk(h, chunks[i], s))) return rc;
   }
   b->drop_graph();   // launch shapes changed
   return DPS_OK;

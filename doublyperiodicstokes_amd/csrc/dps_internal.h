@@ -202,6 +202,9 @@ struct SpreadArgs {
 #define FX_TY 8
 #define FX_BATCH 16          // entries staged together
 #define FX_AMAX_BLOCKS 64
+// passes, each with cell lists of its own: forces; forces and torques
+// (derivative kernels); torques as a vector field (regular kernel)
+enum { FX_FORCES, FX_TORQUES, FX_REGULAR };
 struct FxArgs {
   int N, Nx, Ny, Nz, periodic_z;
   int ZC, ntx, nty, nch;
@@ -219,6 +222,7 @@ struct FxArgs {
   double K0, K1;               // |contribution| <= K0 max|F| + K1 max|T|
   void* grid;
 };
+void launch_fx_lists(const FxArgs& A, hipStream_t s);
 void launch_spread_fx(const FxArgs& A, int words, const double* F, const double* Tq, hipStream_t s);
 
 struct InterpArgs {

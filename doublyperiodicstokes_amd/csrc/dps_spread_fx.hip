@@ -7,7 +7,8 @@
 // SpreadInterpWrapper.cpp:66-107).
 //
 //  k_fx_cells    the (tile, z chunk) cells that a pass's entries reach: counts,
-//                then (after k_fx_scan) the entry lists
+//                then (after k_fx_scan) the entry lists; with the positions, once
+//                a solver has had a product of this pass
 //  k_fx_absmax   partial maxima of |F|, |T| for the fixed-point scale
 //  k_spread_fx   one workgroup per cell, LDS accumulation, one coalesced write
 //                per grid element
@@ -188,7 +189,7 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
   for (int i = threadIdx.x; i < 3 * vol; i += blockDim.x) acc[i] = (TA)0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
-  // this cell's entries, listed when the positions were set
+  // this cell's entries (launch_fx_lists)
   const int e0 = A.start[cell];
   const int ncand = max(0, min(A.start[cell + 1], A.cap) - e0);   // within the list's capacity
   if (wave == 0) {
@@ -470,13 +471,18 @@ size_t fx_lds_bytes(int ZC, int words)
          4 * sizeof(float);
 }
 
-void launch_spread_fx(const FxArgs& A, int words, const double* F, const double* Tq, hipStream_t s)
+void launch_fx_lists(const FxArgs& A, hipStream_t s)
 {
   const int ncells = A.ntx * A.nty * A.nch, ne = A.N * A.nkind;
   hipLaunchKernelGGL(k_fx_zero, dim3((ncells + 255) / 256), dim3(256), 0, s, A.counts, ncells);
   if (ne > 0) hipLaunchKernelGGL(k_fx_cells<false>, dim3((ne + 255) / 256), dim3(256), 0, s, A);
   hipLaunchKernelGGL(k_fx_scan, dim3(1), dim3(1024), 0, s, A.counts, A.start, ncells);
   if (ne > 0) hipLaunchKernelGGL(k_fx_cells<true>, dim3((ne + 255) / 256), dim3(256), 0, s, A);
+}
+
+void launch_spread_fx(const FxArgs& A, int words, const double* F, const double* Tq, hipStream_t s)
+{
+  const int ncells = A.ntx * A.nty * A.nch;
   hipLaunchKernelGGL(k_fx_absmax, dim3(FX_AMAX_BLOCKS), dim3(256), 0, s, F, Tq, 3 * A.N, const_cast<float*>(A.amax));
   const size_t lds = fx_lds_bytes(A.ZC, words);
   const dim3 grid(ncells), block(256);

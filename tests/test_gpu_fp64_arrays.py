@@ -1,0 +1,193 @@
+"""FP64 arrays on mixed-precision solvers: the cell lists of the fixed-point
+spreading are built with the positions (a product at fixed positions launches
+no list kernels), and they follow the positions in every order of eager and
+captured calls.  Integer sums do not depend on their order, so each result
+equals that of a fresh solver at the same positions bit for bit; the spread
+grid agrees with the FP64 oracle to the mixed-precision bound."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_parity import rel_l2, say
+
+pytestmark = pytest.mark.gpu
+
+ETA = 1 / (6 * np.pi)
+N, NX, NZ, LZ = 300, 32, 33, 12.0
+L = 0.5 * NX
+KINDS = ["forces", "torques", "regular"]
+
+
+def _solver(kind):
+    from doublyperiodicstokes_amd import DPStokes, StokesParameters
+    par = StokesParameters(viscosity=ETA, Lx=L, Ly=L, zmin=0.0, zmax=LZ, w=6, w_d=0 if kind == "forces" else 5,
+                           beta=1.785 * 6, beta_d=1.785 * 5, nx=NX, ny=NX, nz=NZ, mode="slit", precision="mixed",
+                           useRegKernel=kind == "regular")
+    s = DPStokes()
+    s.initialize(par, N)
+    return s
+
+
+def _inputs(kind, seed=3):
+    import torch
+    rng = np.random.RandomState(seed)
+    pos = [torch.tensor(np.stack([rng.uniform(0, L, N), rng.uniform(0, L, N), rng.uniform(0.3, LZ - 0.3, N)], 1).ravel(),
+                        device="cuda") for _ in range(4)]
+    F = torch.tensor(rng.normal(size=3 * N), device="cuda")
+    T = None if kind == "forces" else torch.tensor(rng.normal(size=3 * N), device="cuda")
+    return pos, F, T
+
+
+def _fresh(kind, pos, F, T):
+    s = _solver(kind)
+    s.setPositions(pos)
+    out = [None if a is None else a.cpu().numpy() for a in s.mdot_device(F, T)]
+    s.clear()
+    return out
+
+
+def _same(got, want):
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert np.array_equal(a.cpu().numpy(), b)
+
+
+def _kernel_nodes(graph):
+    hip = ctypes.CDLL("libamdhip64.so")
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_products_build_no_lists(kind):
+    """Launches of a captured product: with FP64 arrays those of FP32 arrays
+    and, per spreading pass, the maxima that set the fixed-point scale."""
+    import torch
+    say("launches of a product with FP64 arrays, %s" % kind)
+    pos, F, T = _inputs(kind)
+    count = {}
+    for dt in (torch.float32, torch.float64):
+        s = _solver(kind)
+        s.setPositions(pos[0])
+        f, t = F.to(dt), None if T is None else T.to(dt)
+        s.mdot_device(f, t)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            s.mdot_device(f, t)
+        count[dt] = _kernel_nodes(g)
+        s.clear()
+    say("  FP32 arrays %d, FP64 arrays %d" % (count[torch.float32], count[torch.float64]))
+    assert count[torch.float64] <= count[torch.float32] + (2 if kind == "regular" else 1)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_lists_follow_positions(kind):
+    import torch
+    say("FP64 arrays over changing positions, %s" % kind)
+    pos, F, T = _inputs(kind)
+    want = [_fresh(kind, p, F, T) for p in pos]
+    wantF = [_fresh(kind, p, F, None) for p in pos]
+    s = _solver(kind)
+    for i in (0, 1):
+        s.setPositions(pos[i])
+        _same(s.mdot_device(F, T), want[i])
+        _same(s.mdot_device(F, None), wantF[i])      # another pass at the same positions
+        _same(s.mdot_device(F, T), want[i])
+    work = pos[2].clone()
+    s.update_positions_device(work, None, 0.0)
+    _same(s.mdot_device(F, T), want[2])
+    s.setPositions(pos[3].float())                   # positions in FP32 as well
+    f32 = _fresh(kind, pos[3].float(), F, T)
+    _same(s.mdot_device(F, T), f32)
+    # a captured step (update, product) replayed on changing positions, with
+    # eager products between the replays
+    buf = pos[0].clone()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        s.update_positions_device(buf, None, 0.0, check=False)
+        out = s.mdot_device(F, T)
+    for i in (1, 2, 0, 3):
+        buf.copy_(pos[i])
+        g.replay()
+        torch.cuda.synchronize()
+        _same(out, want[i])
+        _same(s.mdot_device(F, None), wantF[i])
+        _same(s.mdot_device(F, T), want[i])
+    # an eager set, then a replay of a captured product alone
+    gp = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gp):
+        outp = s.mdot_device(F, T)
+    for i in (2, 1):
+        s.setPositions(pos[i])
+        gp.replay()
+        torch.cuda.synchronize()
+        _same(outp, want[i])
+    s.clear()
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_update_captured_before_the_first_product(kind):
+    """A step captured by a solver that had seen FP32 arrays only builds no cell
+    lists: products with FP64 arrays after its replays must not read old ones."""
+    import torch
+    say("update captured before the first product with FP64 arrays, %s" % kind)
+    pos, F, T = _inputs(kind, 5)
+    want = [_fresh(kind, p, F, T) for p in pos]
+    s = _solver(kind)
+    s.setPositions(pos[0])
+    s.mdot_device(F.float(), None if T is None else T.float())
+    buf = pos[0].clone()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        s.update_positions_device(buf, None, 0.0, check=False)
+    _same(s.mdot_device(F, T), want[0])
+    for i in (1, 2, 3):
+        buf.copy_(pos[i])
+        g.replay()
+        _same(s.mdot_device(F, T), want[i])
+        _same(s.mdot_device(F, T), want[i])
+    s.setPositions(pos[1])
+    _same(s.mdot_device(F, T), want[1])
+    s.clear()
+
+
+def test_chunks_change_under_captured_products():
+    """A z chunk set after products were captured -- by the caller, and by two
+    batches that share a solver -- leaves every replay right."""
+    import torch
+    from doublyperiodicstokes_amd import DPStokesBatch
+    from doublyperiodicstokes_amd import _native as Nt
+    say("z chunks changed under captured products")
+    kind = "torques"
+    pos, F, T = _inputs(kind, 7)
+    want = _fresh(kind, pos[0], F, T)
+    ok = lambda out: all(rel_l2(a.cpu().numpy(), b) <= 1e-6 for a, b in zip(out, want))
+    set_chunk = lambda b, c: Nt.check(Nt.load().dps_batch_set_chunks(b._b, (ctypes.c_int * 1)(c), 1, None))
+    s = _solver(kind)
+    s.setPositions(pos[0])
+    b1, b2 = DPStokesBatch([s]), DPStokesBatch([s])
+    first = [[a[0].clone() for a in b.mdot_device([F], [T])] for b in (b1, b2)]
+    assert all(ok(o) for o in first)
+    for c in (8, 16, 12):
+        set_chunk(b1, c)
+        for b in (b2, b1):
+            assert ok([a[0] for a in b.mdot_device([F], [T])])
+        assert ok(s.mdot_device(F, T))
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        out = s.mdot_device(F, T)
+    for c in (16, 8):
+        set_chunk(b1, c)
+        g.replay()
+        torch.cuda.synchronize()
+        assert ok(out) and ok(s.mdot_device(F, T)) and ok([a[0] for a in b2.mdot_device([F], [T])])
+    b1.clear()
+    b2.clear()
+    s.clear()
