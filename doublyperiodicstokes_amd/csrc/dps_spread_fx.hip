@@ -154,7 +154,7 @@ __device__ __forceinline__ int padded(int off, int wx, int wy, int W, int deriv)
 // column of the entry's clipped support (with at most 32 columns the wave
 // splits the rows into phases).  Every grid element of the cell is written to
 // HBM once, coalesced.
-template <int NPF>
+template <int NPF, bool PAIR>
 __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __restrict__ F,
                                                    const double* __restrict__ Tq)
 {
@@ -232,43 +232,44 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
   // header: sup.x, sup.y, sup.z (klo), sup.w (span), f0, f1, f2; paired
   // entries: force support, torque support, force, torque
   const int HO = A.ho;
-  // staging thread (ss, su) loads words su, su+16, ... of entry ss of a batch
+  // Staging thread (ss, su) loads words su, su+16, ... of entry ss of a batch and
+  // word su of its header.  The words' places in the padded record (0, a zero,
+  // past its end) are formed once, 16 bits each, paired entries two to a
+  // register, others kind 0 low and kind 1 high; so all loads of a batch are
+  // issued together.  Formed per batch, with the header's words found among the
+  // record's, the places took 43 registers, a quarter of the wavefronts: slit,
+  // N = 16384, 256^2 x 96, forces and torques, 135 us; so, and with paired and
+  // other entries in kernels of their own, 68.
   const int ss = threadIdx.x >> 4, su = threadIdx.x & 15;
-  auto prefetch = [&](int qb, int nb, T (&v)[NPF]) {
+  constexpr int NAT = PAIR ? (NPF + 1) / 2 : NPF;
+  unsigned at[NAT];
+#pragma unroll
+  for (int k = 0; k < NAT; ++k) {
+    auto place = [&](int off) {   // paired: force record, then torque record
+      return off < A.pm ? padded(off, A.wx0, A.wy0, A.W0, 0)
+                        : (off < A.pm + A.pd ? A.off1 + padded(off - A.pm, A.wx1, A.wy1, A.W1, 1) : 0);
+    };
+    if (PAIR)
+      at[k] = place(su + 32 * k) | (unsigned)place(su + 32 * k + 16) << 16;
+    else
+      at[k] = (su + 16 * k < A.pm ? place(su + 16 * k) : 0) | (unsigned)place(A.pm + su + 16 * k) << 16;
+    asm volatile("" : "+v"(at[k]));
+  }
+  constexpr int NH = PAIR ? 14 : 7;   // header words
+  auto prefetch = [&](int qb, int nb, T (&v)[NPF], T& hd) {
     if (ss >= nb) return;
     const int ent = queue[qb + ss];
     const int p = ent >> 1, kind = ent & 1;
-    if (A.pair) {
-      const T* rm = (const T*)A.rec + (size_t)p * A.rs;
-      const T* rd = rm + A.off1;
-      const int* sm = reinterpret_cast<const int*>(A.sup0 + p);
-      const int* sd = reinterpret_cast<const int*>(A.sup1 + p);
+    const T* rec = (const T*)A.rec + (size_t)p * A.rs;
 #pragma unroll
-      for (int k = 0; k < NPF; ++k) {
-        const int off = su + 16 * k;
-        T xv = (T)0;
-        if (off < A.pm) xv = rm[padded(off, A.wx0, A.wy0, A.W0, 0)];
-        else if (off < A.pm + A.pd) xv = rd[padded(off - A.pm, A.wx1, A.wy1, A.W1, 1)];
-        else if (off >= HO && off < HO + 4) xv = (T)sm[off - HO];
-        else if (off >= HO + 4 && off < HO + 8) xv = (T)sd[off - HO - 4];
-        else if (off >= HO + 8 && off < HO + 11) xv = (T)F[3 * (size_t)p + off - HO - 8];
-        else if (off >= HO + 11 && off < HO + 14) xv = (T)Tq[3 * (size_t)p + off - HO - 11];
-        v[k] = xv;
-      }
-      return;
-    }
-    const int rs = kind ? A.pd : A.pm;
-    const T* rec = (const T*)A.rec + (size_t)p * A.rs + (kind ? A.off1 : 0);
-    const int* sp = reinterpret_cast<const int*>((kind ? A.sup1 : A.sup0) + p);
-    const Tin* fp = (kind ? Tq : F) + 3 * (size_t)p;
-#pragma unroll
-    for (int k = 0; k < NPF; ++k) {
-      const int off = su + 16 * k;
-      T xv = (T)0;
-      if (off < rs) xv = kind ? rec[padded(off, A.wx1, A.wy1, A.W1, 1)] : rec[padded(off, A.wx0, A.wy0, A.W0, 0)];
-      else if (off >= HO && off < HO + 4) xv = (T)sp[off - HO];
-      else if (off >= HO + 4 && off < HO + 7) xv = (T)fp[off - HO - 4];
-      v[k] = xv;
+    for (int k = 0; k < NPF; ++k)
+      v[k] = rec[PAIR ? at[PAIR ? k / 2 : 0] >> 16 * (k & 1) & 0xffff : at[PAIR ? 0 : k] >> (kind ? 16 : 0) & 0xffff];
+    const bool second = PAIR ? su >= 4 : kind;   // the second kernel's support
+    if (su < (PAIR ? 8 : 4)) {
+      hd = (T)reinterpret_cast<const int*>((second ? A.sup1 : A.sup0) + p)[su & 3];
+    } else if (su < NH) {
+      const int c = su - (PAIR ? 8 : 4);
+      hd = (T)((PAIR ? c >= 3 : kind) ? Tq : F)[3 * (size_t)p + (PAIR && c >= 3 ? c - 3 : c)];
     }
   };
   constexpr int QN = 2 * 256;   // queue capacity
@@ -277,15 +278,18 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
     for (int i = threadIdx.x; i < nq_entries; i += blockDim.x) queue[i] = A.entries[e0 + c0 + i];
     __syncthreads();
     // ---- spread the queued entries in staged batches, one wavefront per entry ----
-    T pf[NPF];
-    prefetch(0, min(B, nq_entries), pf);
+    T pf[NPF], ph = 0;
+    prefetch(0, min(B, nq_entries), pf, ph);
     for (int qb = 0; qb < nq_entries; qb += B) {
       const int nb = min(B, nq_entries - qb);
-      if (ss < nb)
+      if (ss < nb) {
 #pragma unroll
-        for (int k = 0; k < NPF; ++k) bst[ss * SLOT + su + 16 * k] = pf[k];
+        for (int k = 0; k < NPF; ++k)
+          if (su + 16 * k < HO) bst[ss * SLOT + su + 16 * k] = pf[k];
+        if (su < NH) bst[ss * SLOT + HO + su] = ph;
+      }
       __syncthreads();
-      if (qb + B < nq_entries) prefetch(qb + B, min(B, nq_entries - qb - B), pf);
+      if (qb + B < nq_entries) prefetch(qb + B, min(B, nq_entries - qb - B), pf, ph);
       for (int si = wave; si < nb; si += nwaves) {
         const T* st = bst + si * SLOT;
         // the entry's header is the same for every lane: scalar registers
@@ -307,7 +311,7 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
         int om = 0, od = 0, spm = 0, spd = 0;
         T t0 = 0, t1 = 0, t2 = 0;
         const T* pd_w = st + A.pm;   // torque record: [wx][wy][dx][dy][z][dz]
-        if (A.pair) {
+        if (PAIR) {
           kind = 2;
           const int klm = klo;
           spm = span;
@@ -330,10 +334,12 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
         const int kls = klo + szp * A.Nz;
         const int qa = max(0, Z0 - kls), qb2 = min(span, Z0 + nZ - kls);
         if (qb2 <= qa) continue;
+#pragma unroll 1   // else nine copies of the point loops: 68 -> 107 us
         for (int sxp = -1; sxp <= 1; ++sxp) {
           int ix0, lx0;
           const int cx = clip_piece(bx, wx, X0, nX, A.Nx, sxp * A.Nx, &ix0, &lx0);
           if (!cx) continue;
+#pragma unroll 1
           for (int syp = -1; syp <= 1; ++syp) {
             int iy0, ly0;
             const int cy = clip_piece(by, wy, Y0, nY, A.Ny, syp * A.Ny, &iy0, &ly0);
@@ -487,8 +493,11 @@ void launch_spread_fx(const FxArgs& A, int words, const double* F, const double*
   const size_t lds = fx_lds_bytes(A.ZC, words);
   const dim3 grid(ncells), block(256);
   switch (words) {
-#define FX_CASE(W) \
-  case W: hipLaunchKernelGGL(k_spread_fx<W>, grid, block, lds, s, A, F, Tq); break;
+#define FX_CASE(W)                                                                                 \
+  case W:                                                                                          \
+    if (A.pair) hipLaunchKernelGGL((k_spread_fx<W, true>), grid, block, lds, s, A, F, Tq);         \
+    else hipLaunchKernelGGL((k_spread_fx<W, false>), grid, block, lds, s, A, F, Tq);               \
+    break;
     FX_CASE(8) FX_CASE(10) FX_CASE(12) FX_CASE(16) FX_CASE(20) FX_CASE(24) FX_CASE(32)
 #undef FX_CASE
     default: break;   // staged_words gives no other

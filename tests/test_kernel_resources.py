@@ -1,7 +1,9 @@
 """Private memory of the built kernels (from the metadata of the gfx950 code
 objects in the library): the FP32 lane-group spectral solve of up to 32 and
 of 49 to 64 levels keeps its rows in registers, none of them in scratch, and
-so do the FFT kernels for radices up to 20 in both precisions."""
+so do the FFT kernels for radices up to 20 in both precisions.  The fixed-point
+spreading stays within 128 registers where its LDS lets four workgroups onto a
+CU (records of up to 153 words)."""
 import os
 import re
 import struct
@@ -31,7 +33,7 @@ def code_objects(data):
 
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    """{demangled kernel name: scratch bytes per lane}."""
+    """{kernel name: (scratch bytes per lane, vector registers)}."""
     llvm = os.path.join(b.ROCM, "llvm", "bin")
     tool = os.path.join(llvm, "llvm-readelf")
     if not os.path.exists(b.lib_path()):
@@ -46,8 +48,9 @@ def kernels(tmp_path_factory):
         path = d / ("%d.co" % i)
         path.write_bytes(image)
         text = subprocess.run([tool, "--notes", str(path)], stdout=subprocess.PIPE, check=True).stdout.decode()
-        for m in re.finditer(r"\.name:\s+(_Z\S*)\n\s+\.private_segment_fixed_size:\s+(\d+)", text):
-            out[m.group(1)] = int(m.group(2))
+        for block in text.split("- .agpr_count:")[1:]:
+            get = lambda key: re.search(r"\.%s:\s+(\S+)" % key, block).group(1)  # noqa: E731
+            out[get("name")] = int(get("private_segment_fixed_size")), int(get("vgpr_count"))
     return out
 
 
@@ -55,12 +58,18 @@ def kernels(tmp_path_factory):
 def test_lane_group_solve_has_no_scratch(kernels, lpm, e):
     found = [v for k, v in kernels.items() if "k_spectralIfLi%dELi%dE" % (lpm, e) in k]
     assert len(found) == 1
-    assert found[0] == 0
+    assert found[0][0] == 0
 
 
 @pytest.mark.parametrize("real", ["f", "d"])
 @pytest.mark.parametrize("rmax", [10, 16, 20])
 def test_fft_kernels_have_no_scratch(kernels, real, rmax):
     for name in ("k_fft_colsI%sLi%dELin1E", "k_fft_colsI%sLi%dELi1E", "k_fft_rows_fwdI%sLi%dE", "k_fft_rows_invI%sLi%dE"):
-        found = [v for k, v in kernels.items() if name % (real, rmax) in k]
+        found = [v[0] for k, v in kernels.items() if name % (real, rmax) in k]
         assert found == [0], name
+
+
+@pytest.mark.parametrize("words", [8, 10])
+def test_fixed_point_spreading_registers(kernels, words):
+    found = [v for k, v in kernels.items() if "k_spread_fxILi%dE" % words in k]
+    assert found and all(scratch == 0 and vgpr <= 128 for scratch, vgpr in found)
