@@ -16,7 +16,7 @@ LIBDIR = os.path.join(HERE, "lib")
 LIBNAME = "libdpstokes_hip.so"
 SOURCES = ["dps_api.hip", "dps_kernels.hip", "dps_spread.hip", "dps_spread_fx.hip",
            "dps_spectral.hip", "dps_chains.hip", "dps_fft.hip", "dps_zgemm.hip"]
-HEADERS = ["dps_core.h", "dps_fft.h", "dps_internal.h", "dps_mma.h", "dps_seg.h", "dps_tables.h"]
+HEADERS = ["dps_core.h", "dps_fft.h", "dps_internal.h", "dps_mma.h", "dps_seg.h", "dps_tables.h", "dps_tune.h"]
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 

@@ -19,6 +19,7 @@
 #include <vector>
 #include "../../include/dpstokes_hip.h"
 #include "dps_internal.h"
+#include "dps_tune.h"
 #include "dps_tables.h"
 
 using namespace dps;
@@ -106,8 +107,9 @@ struct dps_handle {
   ChebTables cheb;
   ChebTransform ct;
   int ntx = 0, nty = 0, ntiles = 0;   // spreading tiles
-  int nt = 1;       // 16-level z tiles per spreading wavefront
-  int ZC = 16;      // z chunk of the spreading as the batch interface names it (rows; nt = its 16-row tiles)
+  int nt = 1;       // 16-level z tiles per spreading wavefront (k_spread)
+  int ZC = 16;      // rows of a fixed-point cell (k_spread_fx)
+  int own_nt = 1, own_zc = 16;   // both as chosen at creation; what a chunk of the batch interface names: chunk_tiles
   int zc_min = 8;   // shortest z chunk the batch interface takes
   size_t lds_max = 65536;   // LDS bytes one workgroup may use on this device
   size_t tsz = 8;   // bytes per grid real
@@ -408,20 +410,7 @@ int build(dps_handle* h)
 // list entries are those of the 16 x 8-column tiles and staged records that
 // the z chunks of the batch interface (dps_batch_set_chunks) are measured in;
 // they stay as they are so that the same solvers and chunks are accepted.
-int staged_words(int rs_max)
-{
-  static const int sizes[] = {8, 10, 12, 16, 20, 24, 32};
-  for (int npf : sizes)
-    if (rs_max + 7 <= 16 * npf) return npf;
-  return 0;
-}
-
-bool chunk_fits(const dps_handle* h, int rs_max, int zc)
-{
-  const int npf = staged_words(rs_max);
-  const size_t bytes = (size_t)3 * zc * (8 * 17 + 1) * h->tsz + (size_t)256 * npf * h->tsz + 2064;
-  return npf > 0 && bytes <= std::min<size_t>(65536, h->lds_max);
-}
+bool chunk_fits(const dps_handle* h, int rs_max, int zc) { return dps::chunk_fits(h->tsz, h->lds_max, rs_max, zc); }
 
 int single_words(const dps_handle* h)
 {
@@ -496,7 +485,8 @@ int build_tiles(dps_handle* h, int wmax)
     h->lds_max = (size_t)lim;
   int rc = check_spread_sizes(h);
   if (rc) return rc;
-  h->nt = spread_tiles(h->Nx, h->Ny, h->Nz, h->prec == DPS_PREC_MIXED);
+  h->nt = h->own_nt = spread_tiles(h->Nx, h->Ny, h->Nz, h->prec == DPS_PREC_MIXED);
+  h->own_zc = h->ZC;
   return DPS_OK;
 }
 
@@ -1978,7 +1968,6 @@ int dps_batch_tune(dps_batch* b, const void* const* forces, const void* const* t
     (void)hipEventDestroy(e0);
     return fail(DPS_ERR_HIP, "event creation failed");
   }
-  static const int cands[] = {8, 16, 32, 48};
   int rc = DPS_OK;
   for (size_t i = 0; i < b->hs.size() && !rc; ++i) {
     dps_handle* h = b->hs[i];
@@ -1986,30 +1975,47 @@ int dps_batch_tune(dps_batch* b, const void* const* forces, const void* const* t
     if (h->N > 0 && !forces[i]) { rc = fail(DPS_ERR_ARG, "null forces"); break; }
     const void* t = torques ? torques[i] : nullptr;
     if (t && !h->has_dip) { rc = fail(DPS_ERR_ARG, "torques given but no dipole kernel (w_d = 0)"); break; }
-    int best = 0, best_nt = h->nt, tried = 0;
-    float best_ms = 1e30f;
-    for (int zc : cands) {
-      // the candidate must be a chunk these inputs' passes take, and one whose
-      // launch differs from the last one's
-      if (zc > h->Nz || zc < h->zc_min || !spread_fits(h, t != nullptr, zc) || (zc + 15) / 16 == tried) continue;
-      tried = (zc + 15) / 16;
-      h->nt = tried;
-      // one untimed call, then the spreading of three calls timed together
-      if ((rc = do_spread(h, forces[i], t, dtype, s))) break;
-      if (hipEventRecord(e0, s) != hipSuccess) { rc = fail(DPS_ERR_HIP, "event record failed"); break; }
-      for (int r = 0; r < 3 && !rc; ++r) rc = do_spread(h, forces[i], t, dtype, s);
-      if (rc) break;
-      float ms = 0;
-      if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-          hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-        rc = fail(DPS_ERR_HIP, "timing failed");
-        break;
+    // the shortest of three timings of three calls of the spreading
+    auto time = [&](float* best) {
+      *best = 1e30f;
+      if ((rc = do_spread(h, forces[i], t, dtype, s))) return;   // untimed
+      for (int k = 0; k < 3; ++k) {
+        if (hipEventRecord(e0, s) != hipSuccess) { rc = fail(DPS_ERR_HIP, "event record failed"); return; }
+        for (int r = 0; r < 3; ++r)
+          if ((rc = do_spread(h, forces[i], t, dtype, s))) return;
+        float ms = 0;
+        if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+            hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
+          rc = fail(DPS_ERR_HIP, "timing failed");
+          return;
+        }
+        *best = std::min(*best, ms);
       }
-      if (ms < best_ms) { best_ms = ms; best = zc; best_nt = h->nt; }
+    };
+    auto fits = [&](int zc) { return zc <= h->Nz && zc >= h->zc_min && spread_fits(h, t != nullptr, zc); };
+    std::vector<float> ms;
+    if (fp64_results(h, dtype)) {
+      // the rows of a cell; a chunk that captured products pin is not varied
+      std::vector<int> cand{h->ZC};
+      if (!h->fx_pinned) cand = chunk_candidates(h->ZC, fits);
+      for (size_t c = 0; c < cand.size() && !rc; ++c) {
+        ms.push_back(1e30f);
+        if (!(rc = set_fx_chunk(h, cand[c], s))) time(&ms.back());
+      }
+      const int rc2 = set_fx_chunk(h, cand[fastest(ms)], s);
+      rc = rc ? rc : rc2;
+      if (chunk_out) chunk_out[i] = h->ZC;
+    } else {
+      const auto cand = tile_candidates(h->nt, h->own_zc, h->own_nt, spread_max_tiles(mixed(h)), fits);
+      for (size_t c = 0; c < cand.size() && !rc; ++c) {
+        ms.push_back(1e30f);
+        h->nt = cand[c].tiles;
+        time(&ms.back());
+      }
+      const SpreadLaunch best = cand[fastest(ms)];
+      h->nt = best.tiles;
+      if (chunk_out) chunk_out[i] = best.chunk;
     }
-    h->nt = best_nt;
-    if (best && !rc) rc = set_fx_chunk(h, best, s);
-    if (chunk_out) chunk_out[i] = h->ZC;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -2035,7 +2041,7 @@ int dps_batch_set_chunks(dps_batch* b, const int* chunks, int torques, void* str
   }
   for (size_t i = 0; i < b->hs.size(); ++i) {
     dps_handle* h = b->hs[i];
-    h->nt = std::max(1, std::min(3, (chunks[i] + 15) / 16));
+    h->nt = chunk_tiles(chunks[i], h->own_zc, h->own_nt, spread_max_tiles(mixed(h)));
     if ((rc = set_fx_chunk(h, chunks[i], s))) return rc;
   }
   b->drop_graph();   // launch shapes changed

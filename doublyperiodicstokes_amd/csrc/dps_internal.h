@@ -182,7 +182,7 @@ struct SpreadArgs {
   int Nx, Ny, Nz;
   int periodic_z;   // rows of a support wrap modulo Nz
   int ntx, nty;
-  int nt;           // 16-level z tiles per wavefront (1..3)
+  int nt;           // 16-level z tiles per wavefront (1..spread_max_tiles)
   int nzg;          // z groups of nt tiles (set by the launcher)
   // particles of every tile (ty ntx + tx), in particle order:
   // lentries[lstart[tile] .. lstart[tile + 1])
@@ -325,6 +325,7 @@ template <class Tin, class T> void launch_stencil(const StencilArgs& A, void* po
 void launch_reset_err(int* e, hipStream_t s);
 // z tiles of 16 levels per spreading wavefront for a grid
 int spread_tiles(int Nx, int Ny, int Nz, bool fp32);
+constexpr int spread_max_tiles(bool fp32) { return fp32 ? 3 : 2; }
 template <class T, class Tin> void launch_spread(const SpreadArgs& A, const void* F, const void* Tq, hipStream_t s);
 template <class T, class Tout> void launch_interp(const InterpArgs& A, void* vel, void* ang, hipStream_t s);
 size_t z_lds_bytes(const ZArgs& A, bool mixed);

@@ -446,7 +446,7 @@ int spread_tiles(int Nx, int Ny, int Nz, bool fp32)
 {
   const long waves = (long)((Nx + 3) / 4) * ((Ny + 3) / 4);
   const int zt = (Nz + 15) / 16;
-  int nt = fp32 ? 3 : 2;
+  int nt = spread_max_tiles(fp32);
   while (nt > 1 && (waves * ((zt + nt - 1) / nt) < 3200 || (zt + nt - 2) / (nt - 1) == (zt + nt - 1) / nt)) --nt;
   return nt;
 }
@@ -467,8 +467,9 @@ void launch_spread(const SpreadArgs& A0, const void* F, const void* Tq, hipStrea
     else hipLaunchKernelGGL((k_spread<T, Tin, false, NT, false>), grid, block, 0, s, A, f, t);          \
     break;
   switch (A.nt) {
-    SPREAD_CASE(1) SPREAD_CASE(2) SPREAD_CASE(3)
-    default: break;   // spread_tiles gives 1..3
+    SPREAD_CASE(1) SPREAD_CASE(2)
+    default:   // three tiles: FP32 grids only
+      if constexpr (sizeof(T) == 4) switch (A.nt) { SPREAD_CASE(3) default: break; }
   }
 #undef SPREAD_CASE
 }

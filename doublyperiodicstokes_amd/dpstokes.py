@@ -373,7 +373,9 @@ class DPStokes:
 
 def tune_key(solver, torques, dtype):
     """Cache key of one batch instance: device architecture, every solver
-    parameter, particle count, whether torques are spread, input dtype."""
+    parameter, particle count, whether torques are spread, input dtype, and
+    the meaning of a chunk ("own": the solver's own chunk names its own launch;
+    choices stored without it were timed on other launches and are not found)."""
     torch = _torch()
     try:
         props = torch.cuda.get_device_properties(solver.device)
@@ -382,7 +384,7 @@ def tune_key(solver, torques, dtype):
         arch = "unknown"
     par = {k: v for k, v in sorted(vars(solver.par).items())}
     return json.dumps({"arch": arch, "par": par, "N": int(solver.N), "torques": bool(torques),
-                       "dtype": str(dtype)}, sort_keys=True, default=str)
+                       "dtype": str(dtype), "chunks": "own"}, sort_keys=True, default=str)
 
 
 def load_tune_cache(path):
@@ -458,6 +460,9 @@ class DPStokesBatch:
 
     def tune(self, forces, torques=None, cache=None):
         """Autotune the spreading z chunk of every instance; returns the chunks.
+        A chunk names the launch of the spreading (the rows of a cell, for FP64
+        arrays on a mixed-precision solver); the launch in use stays unless
+        another is faster.
 
         With ``cache`` (path of a JSON file), instances whose configuration
         the file holds take their stored chunk without timing, provided every

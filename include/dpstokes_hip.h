@@ -203,10 +203,12 @@ int dps_stage_interp(dps_handle* h, const double* grid_in, void* velocities, voi
    dtype replay it with one launch (other pointers re-capture).  Each array
    argument holds one pointer per instance; torques / angular (the arrays or
    their entries) may be NULL.  Position updates of the instances (same
-   buffers) are seen by replays.  dps_batch_tune times the spreading z-chunk
-   candidates of every instance on its current positions and inputs, keeps
-   the fastest (chunk_out: one int per instance, may be NULL) and drops the
-   captured graph. */
+   buffers) are seen by replays.  dps_batch_tune times the spreading of every
+   instance on its current positions and inputs -- the launch in use and the
+   others that a z chunk names; with FP64 arrays on a mixed-precision solver,
+   cells of other heights -- keeps the one in use unless another is faster
+   (chunk_out: the chunk that names it, one int per instance, may be NULL) and
+   drops the captured graph. */
 int dps_batch_create(dps_handle* const* handles, int n, int nstreams, dps_batch** out);
 int dps_batch_destroy(dps_batch* b);
 int dps_batch_mdot(dps_batch* b, const void* const* forces, const void* const* torques, void* const* velocities,
@@ -217,7 +219,9 @@ int dps_batch_tune(dps_batch* b, const void* const* forces, const void* const* t
    dps_batch_tune returned and the caller stored), without timing: each must
    fit its instance (with the torque pass when `torques` is nonzero and the
    instance has a dipole kernel), else DPS_ERR_ARG and nothing changes.
-   Rebuilds the entry lists and drops the captured graph.  No counterpart in
+   Rebuilds the cell lists of FP64 arrays (mixed precision; the cells stay as
+   they are once a graph that the caller captured reads them) and drops the
+   captured graph; other batches of the instances capture again.  No counterpart in
    the reference: it lets a caller reuse tuned choices across runs (the
    Python layer's on-disk tuning cache). */
 int dps_batch_set_chunks(dps_batch* b, const int* chunks, int torques, void* stream);
