@@ -644,30 +644,12 @@ BvpArgs bvp_args(dps_handle* h);
 int allocate_fused(dps_handle* h)
 {
   int rc;
-  const int Nz = h->Nz, NH = h->ct.NH, LPM = h->sp_lpm, E = h->sp_e, R = E / 2;
-  const int NP = (Nz + 1) / 2;   // coefficient pairs (2p, 2p+1)
+  const int Nz = h->Nz, NH = h->ct.NH, LPM = h->sp_lpm, E = h->sp_e;
   const double inv_nxy = 1.0 / ((double)h->Nx * (double)h->Ny);
-  // forward [NH][LPM][E]: coefficient l E + q of node pair j
-  // inverse [NP][LPM][E]: node pair l + LPM r of coefficient 2p (q = r) and
-  // of coefficient 2p+1 (q = R + r)
-  std::vector<double> tf((size_t)NH * LPM * E, 0.0), ti((size_t)NP * LPM * E, 0.0);
-  for (int j = 0; j < NH; ++j)
-    for (int l = 0; l < LPM; ++l)
-      for (int q = 0; q < E; ++q) {
-        const int k = l * E + q;
-        if (k >= Nz) continue;
-        tf[((size_t)j * LPM + l) * E + q] =
-            (k & 1) ? h->ct.TfO[(size_t)(k / 2) * NH + j] : h->ct.TfE[(size_t)(k / 2) * NH + j];
-      }
-  for (int k = 0; k < Nz; ++k)
-    for (int l = 0; l < LPM; ++l)
-      for (int r = 0; r < R; ++r) {
-        const int j = l + LPM * r;
-        if (j >= NH) continue;
-        ti[((size_t)(k / 2) * LPM + l) * E + (k & 1) * R + r] =
-            inv_nxy * ((k & 1) ? h->ct.TiO[(size_t)j * h->ct.NO + k / 2] : h->ct.TiE[(size_t)j * h->ct.NE + k / 2]);
-      }
-
+  h->nzp = chain_rows(Nz);
+  // an FP64 solver solves on chains or on lane groups, a mixed one on both
+  // (run_spectral)
+  const bool lanes = !h->nzp || h->prec == DPS_PREC_MIXED;
   // matrix-core operands in v_mfma 16x16x4 lane order: lane L of step s of row
   // tile t holds row 16 t + L % 16 and term 4 s + L / 16 of the parity's table,
   // zero outside it and for the steps past its terms
@@ -695,7 +677,6 @@ int allocate_fused(dps_handle* h)
     if ((rc = h->upload(&h->d_TfM, cast_vec<float>(fm)))) return rc;
     if ((rc = h->upload(&h->d_TiM, cast_vec<float>(im)))) return rc;
   }
-  h->nzp = chain_rows(Nz);
   if (h->nzp) {
     operands(h->nzp, fm, im);
     if (h->prec == DPS_PREC_MIXED) {
@@ -715,12 +696,35 @@ int allocate_fused(dps_handle* h)
     }
     if ((rc = h->upload(&h->d_ctab, ct))) return rc;
   }
-  if (h->prec == DPS_PREC_MIXED) {
-    if ((rc = h->upload((float**)&h->d_TfP, cast_vec<float>(tf)))) return rc;
-    if ((rc = h->upload((float**)&h->d_TiP, cast_vec<float>(ti)))) return rc;
-  } else {
-    if ((rc = h->upload((double**)&h->d_TfP, tf))) return rc;
-    if ((rc = h->upload((double**)&h->d_TiP, ti))) return rc;
+  if (lanes) {
+    // forward [NH][LPM][E]: coefficient l E + q of node pair j
+    // inverse [NP][LPM][E]: node pair l + LPM r of coefficient 2p (q = r) and
+    // of coefficient 2p+1 (q = R + r)
+    const int R = E / 2, NP = (Nz + 1) / 2;   // coefficient pairs (2p, 2p+1)
+    std::vector<double> tf((size_t)NH * LPM * E, 0.0), ti((size_t)NP * LPM * E, 0.0);
+    for (int j = 0; j < NH; ++j)
+      for (int l = 0; l < LPM; ++l)
+        for (int q = 0; q < E; ++q) {
+          const int k = l * E + q;
+          if (k >= Nz) continue;
+          tf[((size_t)j * LPM + l) * E + q] =
+              (k & 1) ? h->ct.TfO[(size_t)(k / 2) * NH + j] : h->ct.TfE[(size_t)(k / 2) * NH + j];
+        }
+    for (int k = 0; k < Nz; ++k)
+      for (int l = 0; l < LPM; ++l)
+        for (int r = 0; r < R; ++r) {
+          const int j = l + LPM * r;
+          if (j >= NH) continue;
+          ti[((size_t)(k / 2) * LPM + l) * E + (k & 1) * R + r] =
+              inv_nxy * ((k & 1) ? h->ct.TiO[(size_t)j * h->ct.NO + k / 2] : h->ct.TiE[(size_t)j * h->ct.NE + k / 2]);
+        }
+    if (h->prec == DPS_PREC_MIXED) {
+      if ((rc = h->upload((float**)&h->d_TfP, cast_vec<float>(tf)))) return rc;
+      if ((rc = h->upload((float**)&h->d_TiP, cast_vec<float>(ti)))) return rc;
+    } else {
+      if ((rc = h->upload((double**)&h->d_TfP, tf))) return rc;
+      if ((rc = h->upload((double**)&h->d_TiP, ti))) return rc;
+    }
   }
   // The factorisation depends on |k|^2 only: one table entry per distinct
   // value (bit for bit, as ksq_of forms it in the kernels), shared by the
@@ -745,14 +749,16 @@ int allocate_fused(dps_handle* h)
   h->n_fac = nk;
   if ((rc = h->upload(&h->d_fidx, fidx))) return rc;
   const size_t nf = (size_t)nk * E * LPM;
-  if ((rc = h->alloc(&h->d_fib, nf))) return rc;
-  if ((rc = h->alloc(&h->d_fab, nf))) return rc;
-  if ((rc = h->alloc(&h->d_fG, (size_t)nk * 4))) return rc;
+  if (lanes) {
+    if ((rc = h->alloc(&h->d_fib, nf))) return rc;
+    if ((rc = h->alloc(&h->d_fab, nf))) return rc;
+    if ((rc = h->alloc(&h->d_fG, (size_t)nk * 4))) return rc;
+  }
   if (h->nzp)
     if ((rc = h->alloc(&h->d_fJ, (size_t)nk * h->nzp))) return rc;
   double *t_ib = nullptr, *t_ab = nullptr, *t_kq = nullptr;
-  if (hipMalloc((void**)&t_ib, (size_t)(Nz + 1) * nk * sizeof(double)) != hipSuccess ||
-      hipMalloc((void**)&t_ab, (size_t)Nz * nk * sizeof(double)) != hipSuccess ||
+  if ((lanes && (hipMalloc((void**)&t_ib, (size_t)(Nz + 1) * nk * sizeof(double)) != hipSuccess ||
+                 hipMalloc((void**)&t_ab, (size_t)Nz * nk * sizeof(double)) != hipSuccess)) ||
       hipMalloc((void**)&t_kq, (size_t)nk * sizeof(double)) != hipSuccess) {
     if (t_ib) (void)hipFree(t_ib);
     if (t_ab) (void)hipFree(t_ab);
@@ -761,13 +767,13 @@ int allocate_fused(dps_handle* h)
   const BvpArgs A = bvp_args(h);
   hipError_t e0 = hipMemcpy(t_kq, kq.data(), (size_t)nk * sizeof(double), hipMemcpyHostToDevice);
   if (e0 == hipSuccess) {
-    launch_bvp_factor(A.B, t_kq, nk, t_ib, t_ab, LPM, E, h->d_fib, h->d_fab, h->d_fG, 0);
+    if (lanes) launch_bvp_factor(A.B, t_kq, nk, t_ib, t_ab, LPM, E, h->d_fib, h->d_fab, h->d_fG, 0);
     if (h->nzp) launch_chain_factor(A.B, t_kq, nk, h->nzp, h->d_fJ, 0);
   }
   hipError_t e1 = (e0 != hipSuccess) ? e0 : hipGetLastError();
   hipError_t e2 = hipStreamSynchronize(0);
-  (void)hipFree(t_ib);
-  (void)hipFree(t_ab);
+  if (t_ib) (void)hipFree(t_ib);
+  if (t_ab) (void)hipFree(t_ab);
   (void)hipFree(t_kq);
   if (e1 != hipSuccess || e2 != hipSuccess) return fail(DPS_ERR_HIP, "factorisation kernel failed");
   return DPS_OK;
@@ -1436,15 +1442,14 @@ void adjoint_record_sizes(dps_handle* h)
 }
 
 // bytes of the position adjoint's buffers: support records, derivative
-// records, z ranges, second velocity grid, torque second-derivative records
-void adjoint_buffer_bytes(const dps_handle* h, size_t bytes[5])
+// records, second velocity grid, torque second-derivative records
+void adjoint_buffer_bytes(const dps_handle* h, size_t bytes[4])
 {
   const size_t ng = (size_t)3 * h->Nz * h->Ny * h->Nx;
   bytes[0] = (size_t)h->N * sizeof(int4);
   bytes[1] = (size_t)h->N * h->rs_md * h->tsz;
-  bytes[2] = (size_t)h->N * sizeof(int4);
-  bytes[3] = ng * h->tsz;
-  bytes[4] = (size_t)h->N * h->rs_d2 * h->tsz;
+  bytes[2] = ng * h->tsz;
+  bytes[3] = (size_t)h->N * h->rs_d2 * h->tsz;
 }
 
 // buffers of the position adjoint, allocated on its first call
@@ -1453,12 +1458,12 @@ int ensure_adjoint(dps_handle* h)
   if (h->d_gridA) return DPS_OK;
   int rc;
   adjoint_record_sizes(h);
-  size_t b[5];
+  size_t b[4];
   adjoint_buffer_bytes(h, b);
   if ((rc = h->alloc((unsigned char**)&h->d_sup_md, b[0]))) return rc;
   if ((rc = h->alloc((unsigned char**)&h->d_rec_md, b[1]))) return rc;
-  if ((rc = h->alloc((unsigned char**)&h->d_gridA, b[3]))) return rc;
-  if (h->rs_d2 > 0 && (rc = h->alloc((unsigned char**)&h->d_rec_d2, b[4]))) return rc;
+  if ((rc = h->alloc((unsigned char**)&h->d_gridA, b[2]))) return rc;
+  if (h->rs_d2 > 0 && (rc = h->alloc((unsigned char**)&h->d_rec_d2, b[3]))) return rc;
   return DPS_OK;
 }
 
@@ -1758,9 +1763,9 @@ int dps_mdot_adjoint_noalloc(dps_handle* h, const void* forces, const void* torq
     return dps_mdot(h, grad_velocities, grad_angular, grad_forces, grad_torques, dtype, stream);
   }
   adjoint_record_sizes(h);
-  size_t b[5], off[5], need = 0;
+  size_t b[4], off[4], need = 0;
   adjoint_buffer_bytes(h, b);
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < 4; ++i) {
     off[i] = need;
     need += (b[i] + 255) / 256 * 256;
   }
@@ -1778,8 +1783,8 @@ int dps_mdot_adjoint_noalloc(dps_handle* h, const void* forces, const void* torq
   void* rec_d2 = h->d_rec_d2;
   h->d_sup_md = (int4*)(base + off[0]);
   h->d_rec_md = base + off[1];
-  h->d_gridA = base + off[3];
-  h->d_rec_d2 = h->rs_d2 > 0 ? (void*)(base + off[4]) : nullptr;
+  h->d_gridA = base + off[2];
+  h->d_rec_d2 = h->rs_d2 > 0 ? (void*)(base + off[3]) : nullptr;
   rc = adjoint_positions(h, forces, torques, grad_velocities, grad_angular, grad_forces, grad_torques,
                          grad_positions, dtype, (hipStream_t)stream);
   h->d_sup_md = sup_md;

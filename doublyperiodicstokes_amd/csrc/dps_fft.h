@@ -157,7 +157,7 @@ DPS_HD void fft_reg(T (&re)[R], T (&im)[R])
 }
 
 // cos(2 pi m / n) evaluated by the compiler: reduced to an angle of at most
-// pi / 4, then the Taylor series of cosine or sine (16 terms, below an ulp)
+// pi / 4, then the Taylor series of cosine or sine (12 terms, below an ulp)
 constexpr double kPi = 3.14159265358979323846264338327950288;
 constexpr double taylor_cos(double x)
 {
