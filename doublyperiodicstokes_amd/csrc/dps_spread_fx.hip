@@ -1,15 +1,17 @@
 // dps_spread_fx.hip -- spreading of FP64 arrays onto FP32 grids by int32 fixed
-// point, whose sums do not depend on their order.  Callers that take FP64
-// results from a mixed-precision solver hold them to 1e-9 from one release to
-// the next, while the sums of dps_spread.hip round differently at 1e-7 (FP32
-// arrays are held to that); so this pair of types keeps these kernels
+// point, whose sums do not depend on their order.  FP64 results of a
+// mixed-precision solver stay the same to the last bits as before the matrix
+// products, whose sums differ by 1e-7 -- within the accuracy of either, but not
+// within an FP64 comparison with stored results; so this pair of types keeps
+// these kernels
 // (SpreadInterp.cpp:302-448 + BoundaryConditions.h:22-361 +
 // SpreadInterpWrapper.cpp:66-107).
 //
 //  k_fx_cells    the (tile, z chunk) cells that a pass's entries reach: counts,
 //                then (after k_fx_scan) the entry lists; with the positions, once
 //                a solver has had a product of this pass
-//  k_fx_absmax   partial maxima of |F|, |T| for the fixed-point scale
+//  k_fx_absmax   partial maxima of |F|, |T| for the fixed-point scale, and
+//                partial sums for the choice of a finer one
 //  k_spread_fx   one workgroup per cell, LDS accumulation, one coalesced write
 //                per grid element
 #include <hip/hip_runtime.h>
@@ -90,38 +92,44 @@ __global__ void __launch_bounds__(256) k_fx_cells(FxArgs A)
   });
 }
 
-// partial maxima of |F| and |T|; NaN propagates
+// per block: the largest |F| and |T| (NaN propagates), and the sums of squares
+// and numbers of nonzero values of F and T
 __global__ void __launch_bounds__(256) k_fx_absmax(const double* __restrict__ F, const double* __restrict__ Tq, int n3,
-                                                float* __restrict__ out)
+                                                FxStats* __restrict__ out)
 {
-  __shared__ float red[2][4];
-  float fm = 0.0f, tm = 0.0f;
+  __shared__ FxStats red[4];
+  FxStats v{};
+  auto max2 = [](float m, float a) { return (a > m || a != a) ? a : m; };
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n3; i += gridDim.x * 256) {
-    const float a = fabsf((float)F[i]);
-    fm = (a > fm || a != a) ? a : fm;
-    if (Tq) {
-      const float b = fabsf((float)Tq[i]);
-      tm = (b > tm || b != b) ? b : tm;
-    }
+    const double f = F[i], t = Tq ? Tq[i] : 0.0;
+    v.fm = max2(v.fm, fabsf((float)f));
+    v.tm = max2(v.tm, fabsf((float)t));
+    v.f2 += f * f;
+    v.t2 += t * t;
+    v.nf += f != 0;
+    v.nt += t != 0;
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
-    const float a = __shfl_xor(fm, o, 64), b = __shfl_xor(tm, o, 64);
-    fm = (a > fm || a != a) ? a : fm;
-    tm = (b > tm || b != b) ? b : tm;
+    v.fm = max2(v.fm, __shfl_xor(v.fm, o, 64));
+    v.tm = max2(v.tm, __shfl_xor(v.tm, o, 64));
+    v.f2 += __shfl_xor(v.f2, o, 64);
+    v.t2 += __shfl_xor(v.t2, o, 64);
+    v.nf += __shfl_xor(v.nf, o, 64);
+    v.nt += __shfl_xor(v.nt, o, 64);
   }
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = fm;
-    red[1][threadIdx.x >> 6] = tm;
-  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 4; ++w) {
-      fm = (red[0][w] > fm || red[0][w] != red[0][w]) ? red[0][w] : fm;
-      tm = (red[1][w] > tm || red[1][w] != red[1][w]) ? red[1][w] : tm;
+      v.fm = max2(v.fm, red[w].fm);
+      v.tm = max2(v.tm, red[w].tm);
+      v.f2 += red[w].f2;
+      v.t2 += red[w].t2;
+      v.nf += red[w].nf;
+      v.nt += red[w].nt;
     }
-    out[2 * blockIdx.x] = fm;
-    out[2 * blockIdx.x + 1] = tm;
+    out[blockIdx.x] = v;
   }
 }
 
@@ -148,6 +156,76 @@ __device__ __forceinline__ int padded(int off, int wx, int wy, int W, int deriv)
   return off + n;
 }
 
+// A cell's scale from bounds on its columns: the first row of its tile sums, entry
+// by entry (one per thread), the largest |contribution| of the entry at any level
+// of a column, in units four times the present scale's (an entry's bound here is
+// at most 1.5 times the one that scale allows for).
+__device__ __forceinline__ void tight_scale(const FxArgs& A, const double* __restrict__ F, const double* __restrict__ Tq,
+                                         int e0, int ncand, int X0, int Y0, int nX, int nY, int* acc, int RS, int* red,
+                                         float* scl)
+{
+  const float u = 0.25f * scl[0];
+  auto largest = [](const double* v) { return fmaxf(fmaxf(fabsf((float)v[0]), fabsf((float)v[1])), fabsf((float)v[2])); };
+  for (int k = threadIdx.x; k < ncand; k += 256) {
+    const int ent = A.entries[e0 + k], p = ent >> 1, kind = ent & 1;
+    const int4 s = (kind ? A.sup1 : A.sup0)[p];
+    const float* rm = (const float*)A.rec + (size_t)p * A.rs;
+    const float* rd = rm + A.off1;
+    const bool plain = !kind, deriv = kind || A.pair;
+    const RecLayout R = rec_layout(A.wx0, A.wy0, A.W0, 0, 1), D = rec_layout(A.wx1, A.wy1, A.W1, 1, 1);
+    float m = 0, a = 0, b = 0;   // largest z weight; z factors of the x and y derivatives, of the z derivative
+    if (plain) {
+      for (int q = 0; q < A.W0; ++q) m = fmaxf(m, fabsf(rm[R.z + q]));
+      m *= u * largest(F + 3 * (size_t)p);
+    }
+    if (deriv) {
+      for (int q = 0; q < A.W1; ++q) {
+        a = fmaxf(a, fabsf(rd[D.z + q]));
+        b = fmaxf(b, fabsf(rd[D.dz + q]));
+      }
+      const float t = 0.5f * u * largest(Tq + 3 * (size_t)p);
+      a *= t;
+      b *= t;
+    }
+    const int wx = kind ? A.wx1 : A.wx0, wy = kind ? A.wy1 : A.wy0;
+    for (int j = 0; j < wy; ++j) {
+      int y = s.y + j;
+      y += y < 0 ? A.Ny : (y >= A.Ny ? -A.Ny : 0);
+      if ((unsigned)(y - Y0) >= (unsigned)nY) continue;
+      for (int i = 0; i < wx; ++i) {
+        int x = s.x + i;
+        x += x < 0 ? A.Nx : (x >= A.Nx ? -A.Nx : 0);
+        if ((unsigned)(x - X0) >= (unsigned)nX) continue;
+        float v = 0;
+        if (plain) v = fabsf(rm[R.x + i] * rm[R.y + j]) * m;
+        if (deriv)
+          v += (fabsf(rd[D.dx + i] * rd[D.y + j]) + fabsf(rd[D.x + i] * rd[D.dy + j])) * a +
+               fabsf(rd[D.x + i] * rd[D.y + j]) * b;
+        atomicAdd(&acc[(y - Y0) * RS + x - X0], __float2int_ru(v));
+      }
+    }
+  }
+  __syncthreads();
+  int m = 0;
+  for (int i = threadIdx.x; i < FX_TY * RS; i += 256) {
+    m = max(m, acc[i]);
+    acc[i] = 0;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    m = max(max(max(red[0], red[1]), max(red[2], red[3])), 1);
+    int S = 0;
+    (void)frexpf(scl[0], &S);              // the scale is 2^(S - 1)
+    S = min(S - 1 - 2 + __clz(m) - 2, 120);   // 4 m < 2^(34 - clz): partial sums below 2^30 again
+    scl[0] = ldexpf(1.0f, S);
+    scl[1] = ldexpf(1.0f, -S);
+  }
+  __syncthreads();
+}
+
 // One workgroup owns a cell: FX_TX x FX_TY columns and ZC z rows.  Its entries
 // are staged in batches, 16 threads per entry loading record, support and
 // force one batch ahead; a wavefront spreads one entry at a time, a lane per
@@ -170,14 +248,22 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
   // 64-lane instruction per CU, ds_add_f32 ~193, measured on gfx950), and
   // integer sums do not depend on the order of the additions.  The scale 2^S
   // keeps every partial sum below 2^30: a point receives at most one term
-  // per entry of the cell, each at most K0 max|F| + K1 max|T|.
+  // per entry of the cell, each at most K0 max|F| + K1 max|T|.  Where that bound
+  // is far above the sums -- many entries, which do not all meet at one point, or a
+  // few large values among many -- its unit would be too coarse (1500 particles
+  // under one tile: grid 2.8e-5 off; 8000 with one force 100 times the others
+  // 3.3e-3), and the cell's columns are bounded one by one (tight_scale): 1.5e-6 and
+  // 4.1e-6, at 493 and 2837 us a product of either with torques (532 and 2989 with
+  // the coarse unit and the kernel before).
   typedef int TA;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   TA* acc = reinterpret_cast<TA*>(smem_raw);
   const int vol = A.ZC * PL;
   T* bst = reinterpret_cast<T*>(acc + 3 * vol);           // [B][SLOT] staged entries
   int* queue = reinterpret_cast<int*>(bst + B * SLOT);     // p * 2 + kind
-  float* scl = reinterpret_cast<float*>(queue + 2 * 256);  // fixed-point scale and its inverse
+  // fixed-point scale and its inverse; the bound on the cell's sums, and the
+  // root mean square of an entry's
+  float* scl = reinterpret_cast<float*>(queue + 2 * 256);
   T* __restrict__ grid = reinterpret_cast<T*>(A.grid);
   // cells in list order, consecutive cells (the chunks of a tile, then the
   // next tile) on one XCD, whose L2 then holds their shared records
@@ -196,7 +282,7 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
     // the scale: a NaN in the inputs propagates to the whole tile
     float fm = 0.0f, tm = 0.0f;
     for (int i = lane; i < FX_AMAX_BLOCKS; i += 64) {
-      const float a = A.amax[2 * i], b = A.amax[2 * i + 1];
+      const float a = A.stats[i].fm, b = A.stats[i].tm;
       fm = (a > fm || a != a) ? a : fm;
       tm = (b > tm || b != b) ? b : tm;
     }
@@ -213,13 +299,33 @@ __global__ void __launch_bounds__(256) k_spread_fx(FxArgs A, const double* __res
       const int S = min(30 - e, 120);
       scl[0] = ldexpf(1.0f, S);
       scl[1] = isfinite(bound) ? ldexpf(1.0f, -S) : __builtin_nanf("");
+      scl[2] = (float)bound;
     }
+  } else if (wave == 1) {
+    double f2 = 0, t2 = 0;
+    int nf = 0, nt = 0;
+    for (int i = lane; i < FX_AMAX_BLOCKS; i += 64) {
+      f2 += A.stats[i].f2;
+      t2 += A.stats[i].t2;
+      nf += A.stats[i].nf;
+      nt += A.stats[i].nt;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      f2 += __shfl_xor(f2, o, 64);
+      t2 += __shfl_xor(t2, o, 64);
+      nf += __shfl_xor(nf, o, 64);
+      nt += __shfl_xor(nt, o, 64);
+    }
+    if (lane == 0)
+      scl[3] = (float)sqrt((A.K0 * A.K0 * f2 + A.K1 * A.K1 * t2) / max(1, A.pair ? max(nf, nt) : nf + nt));
   }
   // the zeroed accumulator and the scale are complete before any thread adds
   // to the tile or, for a cell without entries, writes it out
   __syncthreads();
   // the scale is folded into each column's coefficients: add takes values
   // already in fixed-point units
+  if (scl[2] > FX_COARSE * scl[3] && isfinite(scl[2])) tight_scale(A, F, Tq, e0, ncand, X0, Y0, nX, nY, acc, RS, queue, scl);
   const T sc = scl[0];
   auto add = [&](TA* d, T v) { atomicAdd(d, __float2int_rn(v)); };
   // z weight q of a row list of n entries, zero outside [0, n): the index
@@ -489,7 +595,7 @@ void launch_fx_lists(const FxArgs& A, hipStream_t s)
 void launch_spread_fx(const FxArgs& A, int words, const double* F, const double* Tq, hipStream_t s)
 {
   const int ncells = A.ntx * A.nty * A.nch;
-  hipLaunchKernelGGL(k_fx_absmax, dim3(FX_AMAX_BLOCKS), dim3(256), 0, s, F, Tq, 3 * A.N, const_cast<float*>(A.amax));
+  hipLaunchKernelGGL(k_fx_absmax, dim3(FX_AMAX_BLOCKS), dim3(256), 0, s, F, Tq, 3 * A.N, const_cast<FxStats*>(A.stats));
   const size_t lds = fx_lds_bytes(A.ZC, words);
   const dim3 grid(ncells), block(256);
   switch (words) {

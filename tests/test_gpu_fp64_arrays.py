@@ -191,3 +191,59 @@ def test_chunks_change_under_captured_products():
     b1.clear()
     b2.clear()
     s.clear()
+
+
+# name, mode, nx, ny, nz, particles, w, w_d, fraction of the box, size of the largest force
+UNEVEN = [
+    ("crowded_tile", "bottom", 64, 32, 33, 1500, 6, 6, 0.04, 1.0),
+    ("crowded_two_kernels", "slit", 64, 32, 33, 1500, 6, 5, 0.06, 1.0),
+    ("crowded_regular", "slit", 64, 32, 33, 1500, 6, 6, 0.05, 1.0),
+    ("crowded_periodic", "periodic", 64, 32, 24, 2500, 5, 5, 0.1, 1.0),
+    ("one_large_force", "slit", 64, 64, 33, 8000, 6, 6, 1.0, 100.0),
+    ("one_large_force_in_a_tile", "bottom", 64, 32, 33, 8000, 6, 0, 0.05, 100.0),
+    ("one_huge_force", "nowall", 48, 40, 30, 900, 5, 4, 1.0, 1e6),
+]
+
+
+@pytest.mark.parametrize("case", UNEVEN, ids=[c[0] for c in UNEVEN])
+def test_crowded_and_uneven_grids(case):
+    """Cells whose bound on the sums is far above them: the spread grid of FP64
+    arrays holds the mixed-precision bound, rel-L2 <= 1e-5, and repeats bit for
+    bit."""
+    import torch
+    from doublyperiodicstokes_amd import DPStokes, StokesParameters
+    from oracle.dp_oracle import OracleDPStokes
+    from oracle.tp_oracle import OracleTPStokes
+    name, mode, nx, ny, nz, n, w, wd, box, top = case
+    say("FP64 arrays, %s" % name)
+    regular = name == "crowded_regular"
+    h = 0.5
+    Lx, Ly, Lz = h * nx, h * ny, (h * nz if mode == "periodic" else 0.35 * nz)
+    rng = np.random.RandomState(n + nx)
+    edge = 0.52 * max(w, wd) * h
+    lo, hi = (edge if mode == "nowall" else 0.1), Lz - (edge if mode in ("nowall", "bottom") else 0.1)
+    pos = np.stack([rng.uniform(0, box * Lx, n), rng.uniform(0, box * Ly, n), rng.uniform(lo, hi, n)], 1).ravel()
+    F = rng.normal(size=3 * n)
+    F[3 * (n // 2):3 * (n // 2) + 3] *= top
+    T = rng.normal(size=3 * n) if wd else None
+    has = wd > 0 and not regular
+    kw = dict(has_torque=has, w_d=wd if has else None, betaw_d=1.785 * wd if has else None)
+    if mode == "periodic":
+        ref = OracleTPStokes(Lx, Ly, 0.0, Lz, nx, ny, nz, ETA, w, 1.785 * w, **kw)
+    else:
+        ref = OracleDPStokes(mode, Lx, Ly, 0.0, Lz, nx, ny, nz, ETA, w, 1.785 * w, **kw)
+    ref.set_positions(pos)
+    par = StokesParameters(viscosity=ETA, Lx=Lx, Ly=Ly, zmin=0.0, zmax=Lz, w=w, w_d=wd, beta=1.785 * w,
+                           beta_d=1.785 * wd if wd else -1.0, nx=nx, ny=ny, nz=nz, mode=mode, precision="mixed",
+                           useRegKernel=regular)
+    s = DPStokes()
+    s.initialize(par, n)
+    s.setPositions(pos)
+    for t in ([None, T] if has else [None]):
+        got = s.stage_spread(torch.from_numpy(F), None if t is None else torch.from_numpy(t)).cpu().numpy()
+        e = rel_l2(got, ref.spread_forces(F, t))
+        say("  %s rel-L2 %.3e" % ("forces" if t is None else "forces and torques", e))
+        assert e <= 1e-5
+        s.setPositions(pos)
+        assert np.array_equal(s.stage_spread(torch.from_numpy(F), None if t is None else torch.from_numpy(t)).cpu().numpy(), got)
+    s.clear()
