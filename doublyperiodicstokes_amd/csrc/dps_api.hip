@@ -1032,8 +1032,8 @@ void build_fx_lists(dps_handle* h, hipStream_t s)
 // A pass is about to read its cell lists: those that the locate built, or, at
 // a pass's first product (and where a replayed locate leaves them out), built
 // here.  The lists depend on the positions alone, so building them in every
-// product would add four launches to each: 17 to 70 us (products at fixed
-// positions, 64x64x30 and 256x256x96).
+// product would add four launches to each: 17 and 30 us (products at fixed
+// positions, 64x64x30 N = 300 and 256x256x96 N = 16384).
 void need_fx_lists(dps_handle* h, int pass, hipStream_t s)
 {
   const unsigned bit = 1u << pass;

@@ -1,13 +1,10 @@
 """Bitwise reproducibility of the mixed-precision path.
 
-With FP32 grids the spreading tile accumulates in int32 fixed point, whose
-sums do not depend on the order in which workgroup threads add; the FFTs,
-the spectral solve and the interpolation's wavefront reductions have fixed
-orders.  So repeated calls on the same inputs give identical bits: the
+The spreading sums run in particle order (each tile's list is sorted); the
+FFTs, the spectral solve and the interpolation's wavefront reductions have
+fixed orders.  So repeated calls on the same inputs give identical bits: the
 spread grid, U and W, for forces only and with torques, with the
-self-mobility's particle on a grid node and for a many-particle slit.  The
-FP64 path accumulates with FP64 LDS atomics, whose order varies; it agrees
-with the oracle to 1e-15 but not bit for bit between calls.
+self-mobility's particle on a grid node and for a many-particle slit.
 """
 import numpy as np
 import pytest
