@@ -28,12 +28,12 @@ def own_chunk(tune, tsz, rs, nz):
     return zc
 
 
-@pytest.mark.parametrize("tsz,max_tiles", [(4, 3), (8, 2)])
-@pytest.mark.parametrize("rs,nz", [(60, 12), (60, 48), (110, 96), (145, 96), (200, 64), (480, 128)])
-def test_tile_candidates(tune, tsz, max_tiles, rs, nz):
+@pytest.mark.parametrize("tsz,rs,nz", [(4, 60, 12), (4, 60, 48), (4, 110, 96), (4, 145, 96), (4, 200, 64),
+                                       (4, 480, 128), (8, 60, 12), (8, 60, 48), (8, 110, 96), (8, 145, 96), (8, 200, 64)])
+def test_tile_candidates(tune, tsz, rs, nz):
+    max_tiles = 3 if tsz == 4 else 2
     own = own_chunk(tune, tsz, rs, nz)
-    if not tune.tune_fits(tsz, rs, own):
-        pytest.skip("no solver of this size")
+    assert tune.tune_fits(tsz, rs, own)
     buf = (ctypes.c_int * 16)()
     for own_tiles in range(1, max_tiles + 1):
         n = tune.tune_tile_candidates(own_tiles, own, own_tiles, max_tiles, tsz, rs, nz, buf)
