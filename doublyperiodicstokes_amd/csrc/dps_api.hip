@@ -140,7 +140,7 @@ struct dps_handle {
   // passes that a captured locate left out: its replays would leave their lists
   // behind, so each of their products builds them
   unsigned fx_lost = 0;
-  // a captured product reads the lists as they are, with its own ZC: ZC stays
+  // a captured product or locate reads or builds lists of the present ZC: ZC stays
   bool fx_pinned = false;
   bool in_batch_capture = false;   // (a batch captures again when ZC changes)
   FxStats* d_fxstats = nullptr;
@@ -1038,16 +1038,14 @@ void need_fx_lists(dps_handle* h, int pass, hipStream_t s)
 {
   const unsigned bit = 1u << pass;
   const bool cap = capturing(s);
-  if (h->fx_on & bit) {
-    if (cap && !h->in_batch_capture) h->fx_pinned = true;
-    return;
-  }
+  if (cap && !h->in_batch_capture) h->fx_pinned = true;
+  if (h->fx_on & bit) return;
   launch_fx_lists(fx_args(h, pass), s);
   if (!cap && !(h->fx_lost & bit)) h->fx_on |= bit;
 }
 
-// z chunk of the fixed-point cells.  It stays as it is where a captured product
-// reads the lists of the present one, or where s only records.
+// z chunk of the fixed-point cells.  It stays as it is where captured calls read
+// or build the lists of the present one, or where s only records.
 int set_fx_chunk(dps_handle* h, int zc, hipStream_t s)
 {
   if (zc == h->ZC || h->fx_pinned) return DPS_OK;
@@ -1082,7 +1080,10 @@ int locate(dps_handle* h, void* positions, int dtype, bool move, const void* vel
   launch_lists(A.L, s);
   if (mixed(h)) {
     build_fx_lists(h, s);
-    if (capturing(s)) h->fx_lost |= ~h->fx_on;
+    if (capturing(s)) {
+      h->fx_lost |= ~h->fx_on;
+      h->fx_pinned |= h->fx_on != 0;
+    }
   }
   HIPCHK(hipGetLastError());
   return DPS_OK;

@@ -220,7 +220,7 @@ int dps_batch_tune(dps_batch* b, const void* const* forces, const void* const* t
    fit its instance (with the torque pass when `torques` is nonzero and the
    instance has a dipole kernel), else DPS_ERR_ARG and nothing changes.
    Rebuilds the cell lists of FP64 arrays (mixed precision; the cells stay as
-   they are once a graph that the caller captured reads them) and drops the
+   they are once a graph that the caller captured uses them) and drops the
    captured graph; other batches of the instances capture again.  No counterpart in
    the reference: it lets a caller reuse tuned choices across runs (the
    Python layer's on-disk tuning cache). */

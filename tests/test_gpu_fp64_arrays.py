@@ -193,6 +193,49 @@ def test_chunks_change_under_captured_products():
     s.clear()
 
 
+@pytest.mark.parametrize("captured", ["first product", "update"])
+def test_chunks_change_under_captured_builds(captured):
+    """A z chunk set after a call that builds cell lists was captured: its
+    replays must not leave lists of another chunk to the eager products."""
+    import torch
+    from doublyperiodicstokes_amd import DPStokesBatch
+    from doublyperiodicstokes_amd import _native as Nt
+    say("z chunks changed after capturing the %s" % captured)
+    kind = "torques"
+    pos, F, T = _inputs(kind, 9)
+    want = [_fresh(kind, p, F, T) for p in pos[:2]]
+    ok = lambda out, i: all(rel_l2(a.cpu().numpy(), b) <= 1e-6 for a, b in zip(out, want[i]))
+    s = _solver(kind)
+    s.setPositions(pos[0])
+    if captured == "update":
+        s.mdot_device(F, T)
+    else:
+        s.mdot_device(F.float(), T.float())
+    buf = pos[0].clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        if captured == "update":
+            s.update_positions_device(buf, None, 0.0, check=False)
+        else:
+            out = s.mdot_device(F, T)
+    b = DPStokesBatch([s])
+    for c in (8, 16, 12, 8):
+        assert ok(s.mdot_device(F, T), 0)
+        Nt.check(Nt.load().dps_batch_set_chunks(b._b, (ctypes.c_int * 1)(c), 1, None))
+        for i in (1, 0):
+            if captured == "update":
+                buf.copy_(pos[i])
+            else:
+                s.setPositions(pos[i])
+            g.replay()
+            torch.cuda.synchronize()
+            assert captured == "update" or ok(out, i)
+            assert ok(s.mdot_device(F, T), i)
+    b.clear()
+    s.clear()
+
+
 # name, mode, nx, ny, nz, particles, w, w_d, fraction of the box, size of the largest force
 UNEVEN = [
     ("crowded_tile", "bottom", 64, 32, 33, 1500, 6, 6, 0.04, 1.0),
